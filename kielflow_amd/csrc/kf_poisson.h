@@ -118,7 +118,10 @@ class Poisson {
     // enqueued between them (Newton-MG; other modes solve in solve_begin):
     // solve_begin enqueues the corrections the last solve needed, solve_end
     // waits for convergence, enqueuing more corrections as needed.
-    void solve_begin(double *phi, const double *rho64, const float *rho32, hipStream_t s, bool from_guess);
+    // fp32_rhs: the solve is part of an FP32 right-hand side, whose transforms'
+    // rounding its potential carries (a direct solve may stop earlier).
+    void solve_begin(double *phi, const double *rho64, const float *rho32, hipStream_t s, bool from_guess,
+                     bool fp32_rhs = false);
     void solve_end();
     PoissonStats last_stats();          // synchronises the stream
     int *device_fail_counter() { return d_fail_; }
@@ -164,7 +167,8 @@ class Poisson {
     template <typename R>
     void zero_level(int l, hipStream_t s);
     template <typename R>
-    void newton_begin(double *phi, const double *rho64, const float *rho32, hipStream_t s, bool from_guess);
+    void newton_begin(double *phi, const double *rho64, const float *rho32, hipStream_t s, bool from_guess,
+                      bool fp32_rhs);
     template <typename R>
     void newton_end();
     template <typename R>
@@ -177,7 +181,7 @@ class Poisson {
         const double *rho64 = nullptr;
         const float *rho32 = nullptr;
         hipStream_t s = nullptr;
-        bool from_guess = false, graph = false, active = false, known = false, direct = false;
+        bool from_guess = false, graph = false, active = false, known = false, direct = false, fp32_rhs = false;
         int it = 0, max_it = 0;
     } run_;
     // BiCGStab on J x = b (level-0 b holds the right side on entry), right

@@ -348,13 +348,14 @@ void Rhs<R>::poisson_begin(const C2<R> *Fn, const C2<R> *staged)
     slot_ = nullptr;
     const double *rho64 = std::is_same<R, double>::value ? (const double *)rho_ : (rho64_on_ ? rho64_ : nullptr);
     const float *rho32 = std::is_same<R, double>::value || rho64_on_ ? nullptr : (const float *)rho_;
+    constexpr bool fp32 = !std::is_same<R, double>::value;
     if (src_ && stage_ >= 0 && !graph_safe_) {
         // a kept potential of this stage (a recomputation of a step whose
         // solve converged before): it passes the first convergence check
         KF_HIP(hipMemcpyAsync(ps_.guess_buffer(), src_[stage_], sizeof(double) * nr, hipMemcpyDeviceToDevice, s_));
         slot_ = ph_[stage_][0];
         ps_.next_guess_converged();
-        ps_.solve_begin(slot_, rho64, rho32, s_, true);
+        ps_.solve_begin(slot_, rho64, rho32, s_, true, fp32);
         return;
     }
     if (stage_ >= 0 && hc_[stage_] >= 2) {
@@ -370,12 +371,12 @@ void Rhs<R>::poisson_begin(const C2<R> *Fn, const C2<R> *staged)
             // the last stage's solution once per step.
             hipLaunchKernelGGL(k_extrap, dim3(nbk(nr)), dim3(256), 0, s_, ps_.guess_buffer(), H, order, nr);
             slot_ = h[0];
-            ps_.solve_begin(slot_, rho64, rho32, s_, true);
+            ps_.solve_begin(slot_, rho64, rho32, s_, true, fp32);
             return;
         }
         hipLaunchKernelGGL(k_extrap, dim3(nbk(nr)), dim3(256), 0, s_, phi_, H, order, nr);
     }
-    ps_.solve_begin(phi_, rho64, rho32, s_, false);
+    ps_.solve_begin(phi_, rho64, rho32, s_, false, fp32);
 }
 
 // convergence of the solve, then the potential history

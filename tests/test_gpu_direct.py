@@ -97,3 +97,34 @@ def test_axis_without_mirror_symmetry_takes_multigrid(ctx):
     phi = g.rfield()
     it, res, code = p.solve(phi, ctx.to_device(rho))
     assert code == kf.api.KF_OK and res <= 1e-10
+
+
+@pytest.mark.parametrize("kind,dims,prec,peak,mean", [
+    ("eqst", (96, 64, 96), "fp64", 1 / 512, 1 / 128), ("eqst", (64, 96, 128), "mixed", 1 / 512, 1 / 128),
+    ("eqst", (24, 24, 24), "fp64", 1 / 512, 1 / 128), ("sist", (64, 48, 64), "fp64", 1 / 128, 1 / 64),
+    ("hyst", (64, 64, 64), "mixed", 1 / 128, 1 / 64)])
+def test_direct_solve_error_is_a_multigrid_solves(ctx, kind, dims, prec, peak, mean):
+    """A direct correction leaves a smooth residual F, whose error is F / e where a V-cycle's rough one is far
+    less: direct solves stop at max|F| <= tol max(peak max|rho|, mean c), c = max(mean e, 0.55 max e), so the
+    error is at most that over min e (maximum principle), and the reference's own, 2e-13 max|rho| / min e."""
+    import kielflow_amd as kf
+    axes = _axes(kind, dims)
+    a = grain_radius(kind, dims[0])
+    for seed in (1, 2, 3):
+        ln_n, nd, _ = kf.setup_host(axes, seed=seed, amp=1e-3, Q=-0.3, a=a)
+        rho = np.exp(ln_n + 0.1 * np.sin(np.arange(dims[1]) * 2 * np.pi / dims[1] + seed)[None, :, None]) + nd
+        out = []
+        for tol in (1e-10, 2e-13):
+            g = kf.Grid(ctx, axes)
+            p = kf.Poisson(g, kf.KF_FP64 if prec == "fp64" or tol < 1e-10 else kf.KF_MIXED, tol=tol, max_it=60)
+            phi = g.rfield()
+            p.solve(phi, ctx.to_device(rho))
+            out.append(phi.get())
+            p.close()
+            g.close()
+        e, top = np.exp(out[1]), np.abs(rho).max()
+        c = max(e.mean(), 0.55 * e.max())
+        bound = (1e-10 * max(peak * top, mean * min(c, top)) + 2e-13 * top) / e.min()
+        err = np.abs(out[0] - out[1]).max()
+        print("direct error", kind, dims, prec, seed, err, "bound", bound, flush=True)
+        assert err <= bound

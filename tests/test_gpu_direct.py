@@ -47,9 +47,8 @@ def test_direct_and_multigrid_corrections_agree(ctx, monkeypatch, kind, dims):
     ln_n, nd, _ = kf.setup_host(axes, seed=2, amp=1e-3, Q=-0.2, a=2.0 * grain_radius(kind, dims[0]))
     rho = np.exp(ln_n) + nd
     tol, out = 1e-11, []
-    for switch in (None, "1"):
-        if switch:
-            monkeypatch.setenv("KF_COARSE_WAVE", switch)
+    for direct in ("1", "0"):
+        monkeypatch.setenv("KF_DIRECT", direct)
         g = kf.Grid(ctx, axes)
         p = kf.Poisson(g, kf.KF_FP64, tol=tol, max_it=60)
         phi = g.rfield()
@@ -128,3 +127,26 @@ def test_direct_solve_error_is_a_multigrid_solves(ctx, kind, dims, prec, peak, m
         err = np.abs(out[0] - out[1]).max()
         print("direct error", kind, dims, prec, seed, err, "bound", bound, flush=True)
         assert err <= bound
+
+
+def test_other_switches_leave_the_corrections_direct(ctx, monkeypatch):
+    """Only KF_DIRECT selects the corrector: a switch of the V-cycle or of the right-hand side, set to any value,
+    changes neither the corrections of a direct solve nor its result."""
+    import kielflow_amd as kf
+    axes = _axes("eqst", (24, 32, 16))
+    ln_n, nd, _ = kf.setup_host(axes, seed=2, amp=1e-3, Q=-0.2, a=2.0)
+    rho, out = ctx.to_device(np.exp(ln_n) + nd), {}
+    for name in ("none", "KF_COARSE_N", "KF_COARSE_WAVE", "KF_PRECOND_COPY", "KF_RHO_STATE", "KF_DIRECT"):
+        if name != "none":
+            monkeypatch.setenv(name, "0" if name == "KF_DIRECT" else "1")
+        g = kf.Grid(ctx, axes)
+        p = kf.Poisson(g, kf.KF_FP64, tol=1e-10, max_it=60)
+        phi = g.rfield()
+        it, _, _ = p.solve(phi, rho)
+        out[name] = (it, phi.get())
+        p.close()
+        g.close()
+        monkeypatch.delenv(name, raising=False)
+    for name in ("KF_COARSE_N", "KF_COARSE_WAVE", "KF_PRECOND_COPY", "KF_RHO_STATE"):
+        assert out[name][0] == out["none"][0] and np.array_equal(out[name][1], out["none"][1]), name
+    assert not np.array_equal(out["KF_DIRECT"][1], out["none"][1])

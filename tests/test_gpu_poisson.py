@@ -65,6 +65,7 @@ def test_wavefront_coarsest_smoothing_gives_identical_results(ctx, monkeypatch, 
     print("coarsest wavefront", kind, n, prec, flush=True)
     axes, _, rho = _problem(kind, n)
     out = []
+    monkeypatch.setenv("KF_DIRECT", "0")
     for wave in ("1", "0"):
         monkeypatch.setenv("KF_COARSE_WAVE", wave)
         g = kf.Grid(ctx, axes)
@@ -89,6 +90,7 @@ def test_preconditioner_on_the_krylov_vectors_gives_identical_results(ctx, monke
     print("preconditioner in place", kind, n, prec, flush=True)
     axes, _, rho = _problem(kind, n)
     out = []
+    monkeypatch.setenv("KF_DIRECT", "0")
     for copy in ("0", "1"):
         monkeypatch.setenv("KF_PRECOND_COPY", copy)
         g = kf.Grid(ctx, axes)

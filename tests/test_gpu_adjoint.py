@@ -276,3 +276,17 @@ def test_checkpointed_run_gradients(ctx):
     assert abs(tM - dM) <= 1e-7 * abs(tM)
     assert abs(tQ - dQ) <= 1e-7 * abs(tQ)
     assert abs(tv - _ip(v, dFn0)) <= 1e-7 * abs(tv)
+
+
+@pytest.mark.parametrize("kind", ["eqst", "sist"])
+def test_adjoint_solve_of_a_nan_is_an_error(ctx, kind):
+    """A NaN in the weight of a velocity reaches every point of the transposed Poisson solve's right-hand side: an error, not a
+    converged solve."""
+    import kielflow_amd as kf
+    g, ps, rhs, phi, S, nd, mask, og = _setup(ctx, kind, 16)
+    w = [np.ones(og.cshape, complex) for _ in range(4)]
+    w[0][1, 2, 3] = np.nan
+    adj = kf.Adjoint(rhs, 1e-3)
+    adj.reset()
+    with pytest.raises(kf.KfError, match="did not converge"):
+        adj.rhs_adjoint([ctx.to_device(s) for s in S], [ctx.to_device(x) for x in w], [g.cfield() for _ in range(4)])

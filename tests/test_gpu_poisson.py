@@ -114,6 +114,38 @@ def test_not_converged_is_an_error(ctx):
     assert code == kf.api.KF_ERR_NOT_CONVERGED
 
 
+@pytest.mark.parametrize("direct", ["1", "0"])
+@pytest.mark.parametrize("kind,prec", [("eqst", "fp64"), ("eqst", "mixed"), ("sist", "fp64"), ("hyst", "mixed")])
+def test_a_residual_that_is_not_a_number_is_a_failure(ctx, monkeypatch, kind, prec, direct):
+    """One NaN or infinity in rho, and a cold start whose first step overshoots the range of exp(phi): a solve
+    that reports convergence has a finite potential and its residual."""
+    import kielflow_amd as kf
+    monkeypatch.setenv("KF_DIRECT", direct)
+    n = 16 if kind == "eqst" else 12
+    axes, _ = axes_for(kind, n)
+    g = kf.Grid(ctx, axes)
+    for name, value in (("nan", np.nan), ("inf", np.inf), ("overshoot", 2000.0)):
+        print("not a number", kind, prec, direct, name, flush=True)
+        rho = np.ones(g.rshape)
+        if name == "overshoot":
+            rho[:] = value
+        else:
+            rho[3, 5, 7] = value
+        p = kf.Poisson(g, kf.KF_FP64 if prec == "fp64" else kf.KF_MIXED, tol=1e-9, max_it=20)
+        phi, drho = g.rfield(), ctx.to_device(rho)
+        it, res, code = p.solve(phi, drho, raise_on_error=False)
+        assert code == kf.api.KF_ERR_NOT_CONVERGED and not res <= 1e-9
+        assert not p.residual(phi, drho) <= 1e-9
+        # the next solve of the same solver is not affected
+        rho[:] = 1.0
+        rho[3, 5, 7] = 1.1
+        phi = g.rfield()
+        it, res, code = p.solve(phi, ctx.to_device(rho))
+        assert code == kf.api.KF_OK and res <= 1e-9 and np.isfinite(phi.get()).all()
+        p.close()
+    g.close()
+
+
 @pytest.mark.parametrize("iters", [1, 3, 25])
 def test_reference_nlj_iterates_match_oracle(ctx, oracle, iters):
     """The reference iteration (Jacobi + damped Newton + Carre SOR), iterate by

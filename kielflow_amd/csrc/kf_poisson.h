@@ -87,10 +87,11 @@ class Poisson {
 
     // J = L_h - diag(exp(phi)) at the given phi (FP64 operator of the adjoint)
     void set_linearization(const double *phi, hipStream_t s);
-    // J x = b to max|b - J x| <= rtol max|b| (FP64; x overwritten; defect
-    // correction with one V-cycle, or two BiCGStab steps on stretched grids,
-    // per iteration).  Returns iterations, or -1 when max_it is reached.
-    // With guess, x holds the initial iterate on entry.
+    // J x = b to max|b - J x| <= rtol max|b| (FP64; x overwritten, and not b;
+    // defect correction by the direct solver, or with one V-cycle, or two
+    // BiCGStab steps on stretched grids, per iteration).  Returns iterations,
+    // or -1 when the last corrector's max_it is reached.  With guess, x holds
+    // the initial iterate on entry.
     int linear_solve(double *x, const double *b, double rtol, int max_it, hipStream_t s, bool guess = false);
     // J^T x = b through  V J V^{-1} = J^T  (V = cell volumes, V L_h symmetric)
     int linear_solve_T(double *x, const double *b, double rtol, int max_it, hipStream_t s, bool guess = false);
@@ -249,7 +250,10 @@ class Poisson {
     double *lsx_ = nullptr, *lsr_ = nullptr;  // linear solve: second iterate, residual
     double *lsT_ = nullptr;  // right-hand side of the transposed solve
     int lin_it_ = 0;
-    int lin_expect_ = 1;          // corrections the last linear solve needed
+    // corrections that the last linear solve took of multigrid [0] and of the
+    // direct solver [1]; direct solves in a row that stalled; solves that
+    // multigrid takes in their place
+    int lin_expect_[2] = {1, 1}, lin_stalls_ = 0, lin_mg_ = 0;
     double *vol_[3] = {};         // per-axis cell volumes (H[i+1]+H[i])/2
     NljState nlj_;
     hipStream_t s0_;

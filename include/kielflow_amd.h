@@ -333,7 +333,12 @@ int kf_batch_box(kf_batch b, int box, double **FUx, double **FUy, double **FUz, 
 /* n_d and solid mask of a box (device FP64 real fields, copied) */
 int kf_batch_set_fields(kf_batch b, int box, const double *nd, const double *mask);
 /* record the graphs; Poisson solves inside run exactly poisson_iterations
- * Newton iterations (unconverged solves are counted as failures) with two
+ * Newton iterations (unconverged solves are counted as failures): direct
+ * corrections followed by as many of multigrid for a replay that they do not
+ * finish, or multigrid alone where direct corrections do not serve (as
+ * kf_poisson_set_smoothing says).  After a replay that needed them, the next
+ * kf_batch_steps waits for that box and records its step again with multigrid
+ * alone; it also waits where a box is 16 steps behind.  Multigrid takes two
  * pre and two post sweeps per level.  The order of the potential warm start
  * (extrapolation in time) is recorded too, so capture needs at least 5
  * kf_batch_steps first, when it is steady (quartic): KF_ERR_ARG otherwise.

@@ -53,8 +53,12 @@ class Batch {
         double2 *F[4] = {};
         double *phi = nullptr;
         hipGraphExec_t exec = nullptr;
+        hipEvent_t ahead = nullptr;  // behind the step AHEAD launches ago
+        long launched = 0;
     };
+    static constexpr int AHEAD = 8;
     void step_box(Box &x);
+    void record(Box &x);
     int precision_;
     double dt_;
     bool captured_ = false;

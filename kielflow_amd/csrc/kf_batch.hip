@@ -26,6 +26,7 @@ Batch::Batch(const std::vector<BatchBox> &boxes, const Switches &sw, int precisi
         for (int d = 0; d < 3; ++d) x->ad[d] = boxes[b].ax[d];
         x->g = new Grid(x->ad, x->s);
         x->ps = new Poisson(x->ad, precision == 1, x->s);
+        KF_HIP(hipEventCreateWithFlags(&x->ahead, hipEventDisableTiming));
         x->ps->init_direct();
         x->ps->set_tolerance(poisson_tol);
         x->ps->set_max_iterations(100);
@@ -55,6 +56,7 @@ Batch::~Batch()
     sync();
     for (Box *x : box_) {
         if (x->exec) (void)hipGraphExecDestroy(x->exec);
+        (void)hipEventDestroy(x->ahead);
         delete x->k32;
         delete x->k64;
         delete x->r32;
@@ -79,6 +81,17 @@ void Batch::set_fields(int b, const double *nd, const double *mask)
 void Batch::step_box(Box &x)
 {
     if (x.exec) {
+        // a replay had to fall back to multigrid, which a recorded direct
+        // solve runs in one workgroup: record the step again, with V-cycles.
+        // At most 2 AHEAD steps of a box are in flight, so that it is seen
+        if (x.ps->captured_direct() && ++x.launched % AHEAD == 0) {
+            KF_HIP(hipEventSynchronize(x.ahead));
+            KF_HIP(hipEventRecord(x.ahead, x.s));
+        }
+        if (x.ps->captured_fell_back()) {
+            KF_HIP(hipStreamSynchronize(x.s));
+            record(x);
+        }
         KF_HIP(hipGraphLaunch(x.exec, x.s));
         return;
     }
@@ -90,6 +103,30 @@ void Batch::steps(int n)
 {
     for (int i = 0; i < n; ++i)
         for (Box *x : box_) step_box(*x);
+}
+
+// one RK4 step of the box into its graph
+void Batch::record(Box &x)
+{
+    hipGraph_t graph = nullptr;
+    KF_HIP(hipStreamBeginCapture(x.s, hipStreamCaptureModeThreadLocal));
+    try {
+        if (x.k32) x.k32->step(x.F);
+        else x.k64->step(x.F);
+    } catch (...) {
+        // leave the stream out of capture mode whatever failed
+        hipGraph_t partial = nullptr;
+        (void)hipStreamEndCapture(x.s, &partial);
+        if (partial) (void)hipGraphDestroy(partial);
+        throw;
+    }
+    KF_HIP(hipStreamEndCapture(x.s, &graph));
+    hipGraphExec_t exec = nullptr;
+    const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    KF_HIP(e);
+    if (x.exec) (void)hipGraphExecDestroy(x.exec);
+    x.exec = exec;
 }
 
 void Batch::capture(int poisson_iterations)
@@ -109,25 +146,7 @@ void Batch::capture(int poisson_iterations)
         // a captured solve runs a fixed number of Newton iterations, so
         // extra sweeps per iteration save nothing: two pre and two post
         x->ps->set_smoothing(2, 2, 24);
-        hipGraph_t graph = nullptr;
-        KF_HIP(hipStreamBeginCapture(x->s, hipStreamCaptureModeThreadLocal));
-        try {
-            if (x->k32) x->k32->step(x->F);
-            else x->k64->step(x->F);
-        } catch (...) {
-            // leave the stream out of capture mode whatever failed
-            hipGraph_t partial = nullptr;
-            (void)hipStreamEndCapture(x->s, &partial);
-            if (partial) (void)hipGraphDestroy(partial);
-            throw;
-        }
-        KF_HIP(hipStreamEndCapture(x->s, &graph));
-        hipError_t e = hipGraphInstantiate(&x->exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        if (e != hipSuccess) {
-            x->exec = nullptr;
-            KF_HIP(e);
-        }
+        record(*x);
     }
     // the capture only recorded the step: nothing advanced
     captured_ = true;

@@ -76,11 +76,17 @@ class Poisson {
     void set_max_iterations(int m) { max_it_ = m; }
     void set_smoothing(int pre, int post, int coarse) { nu1_ = pre; nu2_ = post; nuc_ = coarse; }
     void set_krylov(bool on, int iters) { krylov_ = on; kiters_ = iters; }
-    // k > 0: every Newton-MG solve enqueues exactly k iterations with no
-    // host synchronisation, so a stream capture can record it; iterations
-    // after convergence return at once on the device, and a solve still
-    // unconverged after k counts as a failure.  k = 0: host-driven loop.
+    // k > 0: every Newton-MG solve enqueues k iterations with no host
+    // synchronisation, so a stream capture can record it; iterations after
+    // convergence return at once on the device, and a solve still unconverged
+    // after them counts as a failure.  Direct corrections (where the captured
+    // solve takes them) are followed by k of multigrid for a replay that they
+    // do not finish.  k = 0: host-driven loop.
     void set_graph_iterations(int k) { graph_it_ = k; }
+    // a replay of a captured solve needed multigrid (a new capture records
+    // multigrid alone)
+    bool captured_fell_back() const { return !graph_mg_ && *(volatile int *)(h_ctl_ + FELL) != 0; }
+    bool captured_direct() const { return has_direct() && !graph_mg_; }
     int mode() const { return mode_; }
     double tolerance() const { return tol_; }
     int max_iterations() const { return max_it_; }
@@ -173,7 +179,17 @@ class Poisson {
     template <typename R>
     void newton_end();
     template <typename R>
+    unsigned newton_resid(int it, bool update);
+    template <typename R>
     void newton_check(int it, bool tell);
+    template <typename R>
+    void newton_mg();
+    template <typename R>
+    void newton_run(int n);
+    template <typename R>
+    void newton_fall_back(int budget);
+    template <typename R>
+    void graph_fall_back();
     template <typename R>
     void newton_correct();
     // the Newton solve between newton_begin and newton_end
@@ -184,6 +200,7 @@ class Poisson {
         hipStream_t s = nullptr;
         bool from_guess = false, graph = false, active = false, known = false, direct = false, fp32_rhs = false;
         int it = 0, max_it = 0;
+        int start = 0;  // corrections before multigrid took over
     } run_;
     // BiCGStab on J x = b (level-0 b holds the right side on entry), right
     // preconditioned by one V-cycle; result in level-0 x
@@ -216,6 +233,8 @@ class Poisson {
     long coarse_n_ = 4096;        // levels of at most this many points run in the one-workgroup tail (KF_COARSE_N)
     bool coarse_wave_ = true;     // one wavefront smooths the coarsest level of the tail (KF_COARSE_WAVE=0: all)
     int graph_it_ = 0;
+    bool graph_mg_ = false;       // captures record multigrid
+    static constexpr int FELL = 15;  // slot of h_ctl_
     // direct solver of the shifted operator, of the corrections' precision
     // (init_direct), and the solves that multigrid takes in its place
     Direct<float> *d32_ = nullptr;
@@ -232,7 +251,9 @@ class Poisson {
     int *h_ctl_ = nullptr;
     double *corr64_ = nullptr;    // FP64 scratch (mixed defect correction)
     double *alt64_ = nullptr;     // second potential buffer of the fused Newton update
-    int expect_ = 1;              // corrections the last solve needed (host sync point of the next)
+    // corrections that the last solve took of multigrid [0] and of the direct
+    // solver [1] (host sync point of the next)
+    int expect_[2] = {1, 1};
     bool known_next_ = false;     // the next solve's guess is a converged potential of the same rho
     long n_solves_ = 0, n_corr_ = 0;
     double ion_theta_ = 0.;       // Boltzmann-ion theta (0: none)

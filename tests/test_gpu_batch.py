@@ -4,7 +4,7 @@ stays within 1e-5 of FP64 solo runs."""
 import numpy as np
 import pytest
 
-from helpers import rel_l2
+from helpers import axes_for, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +107,36 @@ def test_batch_capture_needs_full_histories(ctx):
     assert B.poisson_failures() == 0
     B.close()
 
+
+
+@pytest.mark.parametrize("kind,prec", [("eqst", "mixed"), ("eqst", "fp64"), ("sist", "mixed")])
+@pytest.mark.parametrize("start", [0.05, 1.2])
+def test_captured_solves_follow_the_contrast_of_the_density(ctx, kind, prec, start):
+    """The ln n of a box is amp cos(x) with an amplitude that grows by 0.01 a step, so that exp(phi) comes to vary
+    by 3 to 10 over the box, where a direct correction contracts slowly.  A graph recorded with three corrections
+    a solve converges throughout, whether it was recorded before (amp 0.05 at the start) or while (1.2) the
+    contrast was there: its replays fall back to multigrid on the device."""
+    import kielflow_amd as kf
+    print("captured contrast", kind, prec, start, flush=True)
+    n, dt = 24, 1e-3
+    axes = axes_for(kind, n)[0]
+    P = kf.KF_MIXED if prec == "mixed" else kf.KF_FP64
+    B = kf.Batch(ctx, [(axes, kf.api.Parameters(1.0, 0.1, 100.0, 0.0, 0.0))], precision=P, dt=dt, nstreams=1)
+    _, nd, mask = kf.setup_host(axes, seed=3, amp=1e-3, Q=-0.1, a=2.0)
+    B.set_fields(0, ctx.to_device(nd), ctx.to_device(mask))
+    F, phi = B.box(0)
+    x = np.cos(np.arange(n) * 2 * np.pi / n)[:, None, None] + np.zeros((n, n, n))
+    mode = np.fft.rfftn(x)
+    for step in range(6 + 110):
+        if step == 6:
+            B.capture(3)
+            assert B.poisson_failures() == 0
+        F[3].copy_from(ctx.to_device(start * mode if step == 0 else F[3].get() + 0.01 * mode))
+        ctx.sync()
+        B.steps(1)
+        B.sync()
+    e = np.exp(phi.get())
+    print("  exp(phi)", e.min(), e.max(), "failures", B.poisson_failures(), flush=True)
+    assert e.max() / e.min() > 3 and np.isfinite(e).all()
+    assert B.poisson_failures() == 0
+    B.close()

@@ -150,3 +150,49 @@ def test_other_switches_leave_the_corrections_direct(ctx, monkeypatch):
     for name in ("KF_COARSE_N", "KF_COARSE_WAVE", "KF_PRECOND_COPY", "KF_RHO_STATE"):
         assert out[name][0] == out["none"][0] and np.array_equal(out[name][1], out["none"][1]), name
     assert not np.array_equal(out["KF_DIRECT"][1], out["none"][1])
+
+
+def _two_halves(kind, n):
+    rho = np.full((n, n, n), 0.02)
+    rho[: n // 2] = 60.0
+    return _axes(kind, (n, n, n)), rho
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind", ["eqst", "sist"])
+def test_a_budget_that_multigrid_meets_is_met(ctx, monkeypatch, kind, prec):
+    """Corrections that stall do not count against the budget of the multigrid that takes over."""
+    import kielflow_amd as kf
+    axes, rho = _two_halves(kind, 32)
+    budget = 100
+    for direct in ("0", "1"):
+        monkeypatch.setenv("KF_DIRECT", direct)
+        g = kf.Grid(ctx, axes)
+        p = kf.Poisson(g, kf.KF_FP64 if prec == "fp64" else kf.KF_MIXED, tol=1e-9, max_it=budget)
+        phi = ctx.to_device(np.log(rho))
+        it, res, code = p.solve(phi, ctx.to_device(rho))
+        assert code == kf.api.KF_OK and res <= 1e-9
+        if direct == "0":
+            budget = it + 2
+        p.close()
+        g.close()
+
+
+def test_residual_leaves_the_solver_alone(ctx):
+    """kf_poisson_residual between solves does not change which corrector the next ones take."""
+    import kielflow_amd as kf
+    axes, rho = _two_halves("eqst", 32)
+    drho, counts = ctx.to_device(rho), []
+    for between in (False, True):
+        g = kf.Grid(ctx, axes)
+        p = kf.Poisson(g, kf.KF_FP64, tol=1e-9, max_it=100)
+        its = []
+        for _ in range(4):
+            phi = ctx.to_device(np.log(rho))
+            its.append(p.solve(phi, drho)[0])
+            if between:
+                p.residual(phi, drho)
+        counts.append(its)
+        p.close()
+        g.close()
+    assert counts[0] == counts[1] and counts[0][2] < counts[0][0], counts

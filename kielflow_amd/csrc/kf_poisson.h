@@ -233,6 +233,14 @@ class Poisson {
     long coarse_n_ = 4096;        // levels of at most this many points run in the one-workgroup tail (KF_COARSE_N)
     bool coarse_wave_ = true;     // one wavefront smooths the coarsest level of the tail (KF_COARSE_WAVE=0: all)
     int graph_it_ = 0;
+    // the finest level's FP32 x, b, e can be, and are in this solve, stored
+    // colour by colour
+    bool split0_ = false, split_ = false;
+    template <typename R>
+    bool split_level(int l) const
+    {
+        return l == 0 && split_ && std::is_same<R, float>::value;
+    }
     bool graph_mg_ = false;       // captures record multigrid
     static constexpr int FELL = 15;  // slot of h_ctl_
     // direct solver of the shifted operator, of the corrections' precision

@@ -218,3 +218,27 @@ def test_reference_cascade_level_program_matches_oracle(ctx, oracle, program):
         p.set_cascade((-1,), (1,), (1e-3,))               # does not end on the base level
     p.close()
     g.close()
+
+
+@pytest.mark.parametrize("dims", [(32, 24, 16), (16, 32, 12), (64, 64, 64), (48, 96, 192), (12, 32, 64), (24, 48, 6)])
+def test_mixed_vcycles_on_the_colour_split_level(ctx, monkeypatch, dims):
+    """Mixed V-cycles with the finest level stored colour by colour (even extents, Nz a multiple of 4, more than
+    the one-workgroup tail) or not: the potential is the FP64 solve's within both residuals over min e."""
+    import kielflow_amd as kf
+    print("colour split", dims, flush=True)
+    axes = [axes_for("eqst", n)[0][0] for n in dims]
+    ln_n, nd, _ = kf.setup_host(axes, seed=3, amp=1e-3, Q=-0.2, a=2.0 * 16.0 / dims[0])
+    rho = np.exp(ln_n) + nd
+    monkeypatch.setenv("KF_DIRECT", "0")
+    g = kf.Grid(ctx, axes)
+    out = []
+    for prec, tol in ((kf.KF_MIXED, 1e-10), (kf.KF_FP64, 1e-12)):
+        p = kf.Poisson(g, prec, tol=tol, max_it=60)
+        phi = g.rfield()
+        it, res, code = p.solve(phi, ctx.to_device(rho))
+        assert code == kf.api.KF_OK and res <= tol
+        out.append(phi.get())
+        p.close()
+    bound = (1e-10 + 1e-12) * np.abs(rho).max() / np.exp(out[1]).min()
+    assert np.abs(out[0] - out[1]).max() <= bound
+    g.close()

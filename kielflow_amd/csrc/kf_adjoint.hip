@@ -655,7 +655,7 @@ static void r2c_adj(Grid &g, Plan<double> &p, const double *a0, const double *a1
     x.dir = dir;
     x.acc = acc;
     x.coef = coef;
-    if (p.planes) {
+    if (p.plane_fwd) {
         PlaneIn<double> in{};
         in.a0 = four<const double *>(a0);
         in.a1 = four<const double *>(a1);

@@ -292,20 +292,22 @@ void Direct<R>::solve_fourier(const R *b, R *x, const double *c, const int *ctl,
     const long rows = (long)p.nx * p.ny;
     const StridedAddr ay = saddr_y(p);
     const unsigned nv = (unsigned)p.nzc;
-    if (p.planes) {
+    if (p.plane_fwd) {
         plane_r2c<R>(plane_tabs(p), PlaneIn<R>{four<const R *>(b), {}, nullptr, 0, 0}, p.scratch, s, ctl);
-        x_pass(c, ctl, s);
+    } else {
+        launch_zr2c<R>(p.nz / 2, rows, p.tw_m, p.tw_n, Gated<RowLoadReal<R>>{{b, p.nz}, ctl},
+                       RowStoreC<R>{p.scratch, p.nzs}, s, 1000);
+        launch_strided<R, -1>(p.ny, scratch_cols_y(p), p.tw_y, Gated<LoadMasked<R>>{{p.scratch, ay, nv}, ctl},
+                              StoreMasked<R>{p.scratch, ay, nv}, s, 1000, p.vy);
+    }
+    x_pass(c, ctl, s);
+    if (p.plane_inv) {
         PlaneOut<R> z{};
         z.scale = (R)1;
         z.o = four<R *>(x);
         plane_c2r<R>(plane_tabs(p), four<const C2<R> *>(p.scratch), nullptr, nullptr, z, 1, s, ctl);
         return;
     }
-    launch_zr2c<R>(p.nz / 2, rows, p.tw_m, p.tw_n, Gated<RowLoadReal<R>>{{b, p.nz}, ctl},
-                   RowStoreC<R>{p.scratch, p.nzs}, s, 1000);
-    launch_strided<R, -1>(p.ny, scratch_cols_y(p), p.tw_y, Gated<LoadMasked<R>>{{p.scratch, ay, nv}, ctl},
-                          StoreMasked<R>{p.scratch, ay, nv}, s, 1000, p.vy);
-    x_pass(c, ctl, s);
     launch_strided<R, +1>(p.ny, scratch_cols_y(p), p.tw_y, Gated<LoadMasked<R>>{{p.scratch, ay, nv}, ctl},
                           StoreMasked<R>{p.scratch, ay, nv}, s, 1000, p.vy);
     launch_zc2r<R>(p.nz / 2, rows, p.tw_m, p.tw_n, Gated<RowLoadC<R>>{{p.scratch, p.nzs}, ctl},

@@ -403,7 +403,9 @@ struct Plan {
     C2<R> *tw_x = nullptr, *tw_y = nullptr, *tw_m = nullptr, *tw_n = nullptr;
     C2<R> *scratch = nullptr;  // nc complex, for C2R (input is preserved)
     void *owner_pool = nullptr;
-    bool planes = false;       // y and z passes on x planes in LDS (kf_plane.h)
+    // y and z passes on x planes in LDS (kf_plane.h): of several fields in a
+    // launch, and of one field forward, inverse and inverse-and-forward
+    bool planes = false, plane_fwd = false, plane_inv = false, plane_mid = false;
 };
 
 template <typename R>

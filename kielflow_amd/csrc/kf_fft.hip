@@ -153,8 +153,16 @@ void plan_init(Plan<R> &p, int nx, int ny, int nz, hipStream_t s)
     }
     KF_HIP(hipMalloc(&p.scratch, sizeof(C2<R>) * (size_t)nx * ny * p.nzs));
     p.planes = plane_fits(ny, nz / 2, (int)sizeof(C2<R>));
-    // KF_PLANES=0: the separate y and z passes (the same numbers)
-    if (const char *e = std::getenv("KF_PLANES")) p.planes = p.planes && std::atoi(e) != 0;
+    const OnePlane one = plane_one(nx, ny, nz / 2, (int)sizeof(C2<R>));
+    p.plane_fwd = p.planes && one.fwd;
+    p.plane_inv = p.planes && one.inv;
+    p.plane_mid = p.planes && one.mid;
+    // KF_PLANES=0: the separate y and z passes, 1: planes wherever they fit
+    // (the same numbers)
+    if (const char *e = std::getenv("KF_PLANES")) {
+        p.planes = p.planes && std::atoi(e) != 0;
+        p.plane_fwd = p.plane_inv = p.plane_mid = p.planes;
+    }
     autotune(p, s);
 }
 
@@ -173,7 +181,7 @@ template <typename R>
 void r2c(const Plan<R> &p, const R *in, C2<R> *out, hipStream_t s)
 {
     const long rows = (long)p.nx * p.ny;
-    if (p.planes) {
+    if (p.plane_fwd) {
         plane_r2c<R>(plane_tabs(p, p.nzc), PlaneIn<R>{four<const R *>(in), {}, nullptr, 0, 0}, out, s);
         const StridedAddr ax = addr_x(p.nx, p.ny, p.nzc);
         launch_strided<R, -1>(p.nx, (long)p.ny * p.nzc, p.tw_x, LoadPlain<R>{out, ax}, StorePlain<R>{out, ax}, s,
@@ -195,7 +203,7 @@ void c2r(const Plan<R> &p, const C2<R> *in, R *out, hipStream_t s)
     const StridedAddr ax = addr_x(p.nx, p.ny, p.nzc), sy = saddr_y(p);
     launch_strided<R, +1>(p.nx, scratch_cols_x(p), p.tw_x, pad_cols(LoadPlain<R>{in, ax}, p),
                           scratch_store_x(p.scratch, p), s, prof::FFT_X, p.vx);
-    if (p.planes) {
+    if (p.plane_inv) {
         PlaneOut<R> z{};
         z.scale = (R)(1.0 / (double)p.nr);
         z.o = four<R *>(out);

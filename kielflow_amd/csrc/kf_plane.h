@@ -9,7 +9,7 @@
 // numbers are the same bit for bit.
 //
 // Where a plane does not fit, or the lengths are not in the sets below, the
-// separate passes run.  Small grids are bound by the launches, of which an
+// separate passes run; one field's transforms take planes by plane_one.  Small grids are bound by the launches, of which an
 // equidistant evaluation has 7 here in place of 35 and a stretched one 12 in
 // place of 95; at 128^3 FP64 (a plane is 137 KB, one workgroup per CU) the
 // passes over memory still outweigh the idle CUs.  RK4 step, separate passes
@@ -55,6 +55,31 @@ __host__ __device__ constexpr bool plane_fits(int ny, int m, int csize)
 {
     return plane_len_y(ny) && plane_len_m(m) && ny * tpt_for(m) <= 1024 &&
            (ny * (m + 1) + ny + 2 * m + 1) * csize <= 156 * 1024;
+}
+// One field's launch has Nx workgroups, each a whole plane's chain of passes,
+// against launches of its rows and columns: planes of up to `small` bytes are
+// faster whatever Nx is, larger ones from an Nx on.  Separate / plane, us,
+// FP64: forward 128x128 14.5 / 19.6 (Nx = 16), 28.0 / 27.9 (96), 34.1 / 31.5
+// (128), 96x96 17.2 / 18.2 (48), 64x128 16.4 / 14.6 (48); inverse 128x128
+// 13.1 / 19.8 (16), 26.8 / 29.9 (128), 34.6 / 35.2 (256), 96x96 19.1 / 20.5
+// (96), 23.2 / 22.6 (128), 64x128 14.8 / 14.1 (48); a stretched derivative,
+// with its x passes, 128x128 27.4 / 36.9 (16), 49.4 / 51.1 (128), 57.5 / 55.2
+// (192), 96x96 35.4 / 35.3 (48).  FP32: forward 128x128 16.5 / 16.9 (48), 20.1
+// / 19.4 (96), 96x128 14.0 / 12.5 (16); inverse 128x128 25.9 / 27.6 (192), 28.6
+// / 27.8 (256), 96x96 15.6 / 16.3 (96), 17.8 / 17.4 (128), 128x64 12.2 / 14.0
+// (48), 96x64 12.1 / 11.9 (16).
+struct OnePlane {
+    bool fwd, inv, mid;
+};
+inline OnePlane plane_one(int nx, int ny, int m, int csize)
+{
+    const bool dp = csize == 16;
+    const int bytes = ny * (m + 1) * csize;
+    OnePlane o;
+    o.fwd = bytes <= (dp ? 70000 : 60000) || nx >= (dp ? 96 : 64);
+    o.inv = bytes <= (dp ? 70000 : 30000) || (nx >= 128 && bytes <= (dp ? 110000 : 60000)) || nx >= 256;
+    o.mid = bytes <= (dp ? 78000 : 30000) || (nx >= 96 && bytes <= (dp ? 110000 : 60000)) || nx >= 192;
+    return o;
 }
 // threads of a plane's workgroup: its rows' or its columns', whichever are more
 __host__ __device__ constexpr int plane_threads(int ny, int m)

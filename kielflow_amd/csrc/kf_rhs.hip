@@ -338,7 +338,7 @@ void Rhs<R>::poisson_begin(const C2<R> *Fn, const C2<R> *staged)
         z.a0 = nd_;
         z.od = rho64_;
         z.ad = nd64_;
-        if (staged && planes_) yz_c2r<R>(plan_, z, s_, const_cast<C2<R> *>(staged));
+        if (staged && planes_) yz_c2r<R>(plan_, z, s_, staged);
         else if (staged) z_staged<R>(g_, plan_, staged, false, z, s_);
         else c2r_spec<R>(g_, plan_, Fn, 1, -1, z, s_);
     }

@@ -497,24 +497,24 @@ inline bool plane_store(const ZStore<R> &z, PlaneOut<R> &o)
         }
     return false;
 }
-// the inverse y and z passes of the x-transformed buf (scratch layout; the
-// plan's scratch when null) into a ZStore: by planes where the plan has
-// them, else the y pass in place and the z pass
+// the inverse y and z passes of the x-transformed src (scratch layout, kept;
+// the plan's scratch when null) into a ZStore: by planes where the plan takes
+// them for one field, else the y pass into the plan's scratch and the z pass
 template <typename R>
-inline void yz_c2r(Plan<R> &p, const ZStore<R> &st, hipStream_t s, C2<R> *buf = nullptr)
+inline void yz_c2r(Plan<R> &p, const ZStore<R> &st, hipStream_t s, const C2<R> *src = nullptr)
 {
-    C2<R> *b = buf ? buf : p.scratch;
+    const C2<R> *b = src ? src : p.scratch;
     PlaneOut<R> o;
-    if (p.planes && plane_store(st, o)) {
+    if (p.plane_inv && plane_store(st, o)) {
         prof::Scope ps_(prof::FFT_ZC2R, s);
         plane_c2r<R>(plane_tabs(p), four<const C2<R> *>(b), nullptr, nullptr, o, 1, s);
         return;
     }
     const StridedAddr ay = saddr_y(p);
     launch_strided<R, +1>(p.ny, scratch_cols_y(p), p.tw_y, LoadMasked<R>{b, ay, (unsigned)p.nzc},
-                          StoreMasked<R>{b, ay, (unsigned)p.nzc}, s, prof::FFT_Y, p.vy);
+                          StoreMasked<R>{p.scratch, ay, (unsigned)p.nzc}, s, prof::FFT_Y, p.vy);
     with_zstore<R>(st, [&](const auto &z) {
-        launch_zc2r<R>(p.nz / 2, (long)p.nx * p.ny, p.tw_m, p.tw_n, RowLoadC<R>{b, p.nzs}, z, s);
+        launch_zc2r<R>(p.nz / 2, (long)p.nx * p.ny, p.tw_m, p.tw_n, RowLoadC<R>{p.scratch, p.nzs}, z, s);
     });
 }
 template <typename R>
@@ -967,7 +967,7 @@ inline void zprof(Plan<R> &p, C2<R> *buf, const R *kz, const R *prof, int pdir, 
 template <typename R>
 inline void metric_yzy(Plan<R> &p, const R *prof, int b, hipStream_t s)
 {
-    if (p.planes) {
+    if (p.plane_mid) {
         prof::Scope ps_(prof::FFT_ZC2R, s);
         PlaneProf<R> a{};
         a.dst = p.scratch;
@@ -1060,7 +1060,7 @@ inline void z_staged(Grid &g, Plan<R> &p, const C2<R> *H, bool dz, const ZStore<
 template <typename R, typename RS>
 inline void zy_r2c(Plan<R> &p, const RS *src, hipStream_t s)
 {
-    if (p.planes) {
+    if (p.plane_fwd) {
         prof::Scope ps_(prof::FFT_ZR2C, s);
         PlaneIn<R> in{};
         if constexpr (std::is_same<R, RS>::value) in.a0 = four<const R *>(src);

@@ -17,7 +17,10 @@ DIMS = [(16, 16, 16), (12, 24, 32), (6, 16, 192), (24, 128, 16), (16, 48, 96), (
 
 def _eval(ctx, monkeypatch, kind, dims, prec, planes, steps=0):
     import kielflow_amd as kf
-    monkeypatch.setenv("KF_PLANES", planes)
+    if planes is None:
+        monkeypatch.delenv("KF_PLANES", raising=False)
+    else:
+        monkeypatch.setenv("KF_PLANES", planes)
     rng = np.random.default_rng(7)
     axes = [axes_for(kind, n)[0][0] for n in dims]
     g = kf.Grid(ctx, axes)
@@ -37,7 +40,7 @@ def _eval(ctx, monkeypatch, kind, dims, prec, planes, steps=0):
         rhs.solve(0.0, F)
     assert rhs.poisson_failures() == 0
     out = [f.get() for f in F] + [phi.get()]
-    monkeypatch.delenv("KF_PLANES")
+    monkeypatch.delenv("KF_PLANES", raising=False)
     return out
 
 
@@ -49,6 +52,19 @@ def test_plane_passes_give_identical_results(ctx, monkeypatch, kind, dims, prec)
     print("planes", kind, dims, prec, flush=True)
     a = _eval(ctx, monkeypatch, kind, dims, prec, "1")
     b = _eval(ctx, monkeypatch, kind, dims, prec, "0")
+    for name, x, y in zip(["FUx", "FUy", "FUz", "Fn", "phi"], a, b):
+        assert np.isfinite(x).all() and np.array_equal(x, y), (name, float(np.abs(x - y).max()))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind", ["eqst", "sist"])
+@pytest.mark.parametrize("dims", [(8, 128, 128), (64, 96, 96), (96, 96, 96), (128, 128, 64)])
+def test_the_rule_for_one_field_gives_identical_results(ctx, monkeypatch, kind, dims, prec):
+    """Without the switch a field's own forward and inverse passes take planes or not by Nx and the plane's bytes,
+    each for itself, beside the launches of several fields: the same bits as planes throughout."""
+    print("plane rule", kind, dims, prec, flush=True)
+    a = _eval(ctx, monkeypatch, kind, dims, prec, None)
+    b = _eval(ctx, monkeypatch, kind, dims, prec, "1")
     for name, x, y in zip(["FUx", "FUy", "FUz", "Fn", "phi"], a, b):
         assert np.isfinite(x).all() and np.array_equal(x, y), (name, float(np.abs(x - y).max()))
 

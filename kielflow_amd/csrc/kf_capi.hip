@@ -549,7 +549,7 @@ int kf_poisson_create(kf_grid g, int precision, int mode, kf_poisson *out)
         set_dev(g->ctx);
         std::unique_ptr<Poisson> p(new Poisson(g->g->ax, precision == KF_MIXED, g->ctx->stream));
         p->set_mode(mode);
-        if (mode == KF_POISSON_NEWTON_MG) p->init_direct();
+        if (mode == KF_POISSON_NEWTON_MG) p->init_direct(g->p64);
         *out = new kf_poisson_s{g, p.release(), PoissonStats{0, 0., 0}, nullptr};
         return KF_OK;
     });

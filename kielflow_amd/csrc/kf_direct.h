@@ -32,7 +32,8 @@ template <typename R>
 class Direct {
   public:
     // h[d][i] = x_i - x_{i-1}, i = 0..n_d (the solver's spacings)
-    Direct(const AxisDesc ax[3], const std::vector<double> h[3], hipStream_t s);
+    // like: a plan of the grid's lengths that is there already, or null
+    Direct(const AxisDesc ax[3], const std::vector<double> h[3], hipStream_t s, const fft::Plan<R> *like = nullptr);
     ~Direct();
     Direct(const Direct &) = delete;
     Direct &operator=(const Direct &) = delete;

@@ -138,7 +138,7 @@ bool Direct<R>::possible(const AxisDesc ax[3], const std::vector<double> h[3])
 }
 
 template <typename R>
-Direct<R>::Direct(const AxisDesc ax[3], const std::vector<double> h[3], hipStream_t s)
+Direct<R>::Direct(const AxisDesc ax[3], const std::vector<double> h[3], hipStream_t s, const fft::Plan<R> *like)
 {
     fourier_ = true;
     for (int d = 0; d < 3; ++d) {
@@ -191,7 +191,7 @@ Direct<R>::Direct(const AxisDesc ax[3], const std::vector<double> h[3], hipStrea
         fwd_[d] = pool_ + at[3 + d];
         inv_[d] = pool_ + at[6 + d];
     }
-    if (fourier_) plan_init<R>(plan_, n_[0], n_[1], n_[2], s);
+    if (fourier_) plan_init<R>(plan_, n_[0], n_[1], n_[2], s, like, false);
     else KF_HIP(hipMalloc(&tmp_, sizeof(R) * (size_t)n_[0] * n_[1] * n_[2]));
 }
 

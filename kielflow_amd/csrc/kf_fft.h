@@ -408,8 +408,11 @@ struct Plan {
     bool planes = false, plane_fwd = false, plane_inv = false, plane_mid = false;
 };
 
+// like: a plan of the same lengths whose measured choices this one takes;
+// tune_x false: for a caller without strided x passes (and with no y passes
+// of one field, nothing is measured)
 template <typename R>
-void plan_init(Plan<R> &p, int nx, int ny, int nz, hipStream_t s);
+void plan_init(Plan<R> &p, int nx, int ny, int nz, hipStream_t s, const Plan<R> *like = nullptr, bool tune_x = true);
 template <typename R>
 void plan_free(Plan<R> &p);
 

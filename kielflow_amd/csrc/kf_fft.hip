@@ -61,7 +61,7 @@ static C2<R> *twiddles(int n, int count, hipStream_t s)
 // every choice, for tests).  Every choice computes the same numbers; only
 // the speed changes.
 template <typename R>
-static void autotune(Plan<R> &p, hipStream_t s)
+static void autotune(Plan<R> &p, hipStream_t s, bool tune_x)
 {
     p.vx = p.vy = 0;
     const char *env = std::getenv("KF_FFT_AUTOTUNE");
@@ -72,6 +72,7 @@ static void autotune(Plan<R> &p, hipStream_t s)
         p.nzs = p.nzc;
         return;
     }
+    if (!tune_x && p.plane_fwd && p.plane_inv) return;
     KF_HIP(hipMemsetAsync(p.scratch, 0, sizeof(C2<R>) * (size_t)p.nx * p.ny * p.nzs, s));
     hipEvent_t e0, e1;
     KF_HIP(hipEventCreate(&e0));
@@ -126,13 +127,13 @@ static void autotune(Plan<R> &p, hipStream_t s)
     p.nzs = best_nzs;
     p.vy = best_vy;
     ax = saddr_x(p);
-    if (cb_variant<R>(p.nx, 1) != cb_variant<R>(p.nx, 0)) p.vx = time_pass(0, 1) < 0.95f * time_pass(0, 0) ? 1 : 0;
+    if (tune_x && cb_variant<R>(p.nx, 1) != cb_variant<R>(p.nx, 0)) p.vx = time_pass(0, 1) < 0.95f * time_pass(0, 0) ? 1 : 0;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
 }
 
 template <typename R>
-void plan_init(Plan<R> &p, int nx, int ny, int nz, hipStream_t s)
+void plan_init(Plan<R> &p, int nx, int ny, int nz, hipStream_t s, const Plan<R> *like, bool tune_x)
 {
     if (!grid_supported(nx, ny, nz))
         throw Error("grid " + std::to_string(nx) + "x" + std::to_string(ny) + "x" +
@@ -163,7 +164,13 @@ void plan_init(Plan<R> &p, int nx, int ny, int nz, hipStream_t s)
         p.planes = p.planes && std::atoi(e) != 0;
         p.plane_fwd = p.plane_inv = p.plane_mid = p.planes;
     }
-    autotune(p, s);
+    if (like && like->nx == nx && like->ny == ny && like->nz == nz) {
+        p.vx = like->vx;
+        p.vy = like->vy;
+        p.nzs = like->nzs;
+    } else {
+        autotune(p, s, tune_x);
+    }
 }
 
 template <typename R>
@@ -217,8 +224,8 @@ void c2r(const Plan<R> &p, const C2<R> *in, R *out, hipStream_t s)
                    RowStoreReal<R>{out, p.nz, (R)(1.0 / (double)p.nr)}, s);
 }
 
-template void plan_init<float>(Plan<float> &, int, int, int, hipStream_t);
-template void plan_init<double>(Plan<double> &, int, int, int, hipStream_t);
+template void plan_init<float>(Plan<float> &, int, int, int, hipStream_t, const Plan<float> *, bool);
+template void plan_init<double>(Plan<double> &, int, int, int, hipStream_t, const Plan<double> *, bool);
 template void plan_free<float>(Plan<float> &);
 template void plan_free<double>(Plan<double> &);
 template void r2c<float>(const Plan<float> &, const float *, float2 *, hipStream_t);

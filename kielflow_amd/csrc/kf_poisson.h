@@ -71,7 +71,8 @@ class Poisson {
     // the grid admits it; multigrid takes them elsewhere, with Boltzmann
     // ions, and from where a direct correction leaves too much (exp(phi)
     // varies by more than a few times over the box)
-    void init_direct();
+    // (like: an FP64 plan of the grid that is there already, or null)
+    void init_direct(const fft::Plan<double> *like = nullptr);
     void set_tolerance(double t) { tol_ = t; }
     void set_max_iterations(int m) { max_it_ = m; }
     void set_smoothing(int pre, int post, int coarse) { nu1_ = pre; nu2_ = post; nuc_ = coarse; }

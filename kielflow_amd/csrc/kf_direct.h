@@ -47,6 +47,7 @@ class Direct {
     void solve(const R *b, R *x, const double *c, const int *ctl, hipStream_t s);
 
   private:
+    void release();
     void solve_fourier(const R *b, R *x, const double *c, const int *ctl, hipStream_t s);
     void x_pass(const double *c, const int *ctl, hipStream_t s);
     void solve_modal(const R *b, R *x, const double *c, const int *ctl, hipStream_t s);

@@ -12,15 +12,16 @@ using namespace fft;
 // ======================================================================== one axis' modes (host)
 // Eigenvalues of a symmetric tridiagonal matrix (diagonal a, off-diagonal b)
 // and its eigenvectors as the rows of Z, by the implicit QR algorithm with
-// Wilkinson's shift (Golub and Van Loan, Matrix Computations, 8.3).
-static void tridiagonal_modes(std::vector<double> &a, std::vector<double> &b, std::vector<double> &Z)
+// Wilkinson's shift (Golub and Van Loan, Matrix Computations, 8.3).  False
+// when it does not converge.
+static bool tridiagonal_modes(std::vector<double> &a, std::vector<double> &b, std::vector<double> &Z)
 {
     const int m = (int)a.size();
     Z.assign((size_t)m * m, 0.);
     for (int i = 0; i < m; ++i) Z[(size_t)i * m + i] = 1.;
     int hi = m - 1;
     for (long guard = 0; hi > 0; ++guard) {
-        if (guard > 60L * m) throw Error("the axis' eigenvalues did not converge");
+        if (guard > 60L * m) return false;
         for (int i = 0; i < hi; ++i)
             if (std::fabs(b[i]) <= 1.2e-16 * (std::fabs(a[i]) + std::fabs(a[i + 1]))) b[i] = 0.;
         while (hi > 0 && b[hi - 1] == 0.) --hi;
@@ -51,6 +52,7 @@ static void tridiagonal_modes(std::vector<double> &a, std::vector<double> &b, st
             }
         }
     }
+    return true;
 }
 
 static bool mirrored(const std::vector<double> &h, int n)
@@ -67,6 +69,7 @@ static bool mirrored(const std::vector<double> &h, int n)
 // modes (u_{n-i} = u_i) and odd ones, each a tridiagonal matrix.
 struct Modes {
     std::vector<double> lam, T, Ti;  // T[i][m], Ti[m][i]
+    bool ok = true;
 };
 static Modes axis_modes(const std::vector<double> &hin, int n)
 {
@@ -107,7 +110,7 @@ static Modes axis_modes(const std::vector<double> &hin, int n)
         std::vector<double> a(m), b(std::max(m - 1, 0)), Z;
         for (int q = 0; q < m; ++q) a[q] = dot(ks[q], ks[q]);
         for (int q = 0; q + 1 < m; ++q) b[q] = dot(ks[q], ks[q + 1]);
-        tridiagonal_modes(a, b, Z);
+        M.ok = tridiagonal_modes(a, b, Z) && M.ok;
         for (int e = 0; e < m; ++e) {
             const size_t mode = M.lam.size();
             M.lam.push_back(std::min(a[e], 0.));
@@ -170,6 +173,7 @@ Direct<R>::Direct(const AxisDesc ax[3], const std::vector<double> h[3], hipStrea
             for (int e = 0; e < d; ++e)
                 if (h[e] == h[d]) same = e;
             M[d] = same >= 0 ? M[same] : axis_modes(h[d], n_[d]);
+            if (!M[d].ok) throw Error("the axis' eigenvalues did not converge");
             put(d, M[d].lam);
             const int n = n_[d];
             if (d == 2) {
@@ -183,20 +187,31 @@ Direct<R>::Direct(const AxisDesc ax[3], const std::vector<double> h[3], hipStrea
             put(6 + d, M[d].T);
         }
     }
-    KF_HIP(hipMalloc(&pool_, sizeof(R) * host.size()));
-    KF_HIP(hipMemcpyAsync(pool_, host.data(), sizeof(R) * host.size(), hipMemcpyHostToDevice, s));
-    KF_HIP(hipStreamSynchronize(s));
-    for (int d = 0; d < 3; ++d) {
-        lam_[d] = pool_ + at[d];
-        fwd_[d] = pool_ + at[3 + d];
-        inv_[d] = pool_ + at[6 + d];
+    try {
+        KF_HIP(hipMalloc(&pool_, sizeof(R) * host.size()));
+        KF_HIP(hipMemcpyAsync(pool_, host.data(), sizeof(R) * host.size(), hipMemcpyHostToDevice, s));
+        KF_HIP(hipStreamSynchronize(s));
+        for (int d = 0; d < 3; ++d) {
+            lam_[d] = pool_ + at[d];
+            fwd_[d] = pool_ + at[3 + d];
+            inv_[d] = pool_ + at[6 + d];
+        }
+        if (fourier_) plan_init<R>(plan_, n_[0], n_[1], n_[2], s, like, false);
+        else KF_HIP(hipMalloc(&tmp_, sizeof(R) * (size_t)n_[0] * n_[1] * n_[2]));
+    } catch (...) {
+        release();
+        throw;
     }
-    if (fourier_) plan_init<R>(plan_, n_[0], n_[1], n_[2], s, like, false);
-    else KF_HIP(hipMalloc(&tmp_, sizeof(R) * (size_t)n_[0] * n_[1] * n_[2]));
 }
 
 template <typename R>
 Direct<R>::~Direct()
+{
+    release();
+}
+
+template <typename R>
+void Direct<R>::release()
 {
     if (fourier_) plan_free<R>(plan_);
     (void)hipFree(pool_);
@@ -350,9 +365,10 @@ struct ModalMap {
 };
 
 // One wavefront forms a (16 TM) x (16 TN) tile on the matrix cores straight
-// from global memory: the matrix (at most 256 KB) and the field panel are
-// read by neighbouring wavefronts of one XCD, so they come from its L2, and
-// nothing needs a barrier.  At 128^3 FP64 a product is 18.9 us for 0.54
+// from global memory: the matrix (n^2 values: 128 KB at 128 points FP64, 512
+// KB at 256, 2 MB at the 512 of the longest z axis, of a 4 MB L2) and the
+// field panel are read by neighbouring wavefronts of one XCD, so they come
+// from its L2, and nothing needs a barrier.  At 128^3 FP64 a product is 18.9 us for 0.54
 // GFLOP (28 of 72 TFLOP/s that a large FP64 product reaches; its 34 MB stay
 // in the caches), at 64^3 4.7 us, where the launch bounds it.  k is contracted in an order that lets a lane
 // load 16 bytes of A at once: lane group g takes k = KV g .. KV g + KV - 1

@@ -40,7 +40,7 @@ def _sources():
                 yield os.path.join(root, f)
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference tree not mounted")
+@pytest.mark.skipif(not os.path.isdir(REF) or not os.listdir(REF), reason="reference tree not mounted")
 def test_reference_citations_are_in_range():
     idx = _ref_index()
     own = _own_files()

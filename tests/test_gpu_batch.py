@@ -109,6 +109,33 @@ def test_batch_capture_needs_full_histories(ctx):
 
 
 
+def _grow_contrast(kf, ctx, kind, dims, prec, start, steps):
+    """A captured box whose ln n is amp cos(x), amp growing by 0.01 a step from `start`: (min, max of exp(phi),
+    failed solves)."""
+    axes = [axes_for(kind, n)[0][0] for n in dims]
+    P = kf.KF_MIXED if prec == "mixed" else kf.KF_FP64
+    B = kf.Batch(ctx, [(axes, kf.api.Parameters(1.0, 0.1, 100.0, 0.0, 0.0))], precision=P, dt=1e-3, nstreams=1)
+    _, nd, mask = kf.setup_host(axes, seed=3, amp=1e-3, Q=-0.1, a=2.0)
+    B.set_fields(0, ctx.to_device(nd), ctx.to_device(mask))
+    F, phi = B.box(0)
+    mode = np.fft.rfftn(np.cos(np.arange(dims[0]) * 2 * np.pi / dims[0])[:, None, None] + np.zeros(dims))
+    for step in range(steps):
+        if step == 6:
+            B.capture(3)
+            assert B.poisson_failures() == 0
+        d = ctx.to_device(start * mode if step == 0 else F[3].get() + 0.01 * mode)
+        F[3].copy_from(d)
+        ctx.sync()
+        d.free()
+        B.steps(1)
+        B.sync()
+    e, failures = np.exp(phi.get()), B.poisson_failures()
+    print("  exp(phi)", e.min(), e.max(), "failures", failures, flush=True)
+    B.close()
+    assert np.isfinite(e).all()
+    return e.min(), e.max(), failures
+
+
 @pytest.mark.parametrize("kind,prec", [("eqst", "mixed"), ("eqst", "fp64"), ("sist", "mixed")])
 @pytest.mark.parametrize("start", [0.05, 1.2])
 def test_captured_solves_follow_the_contrast_of_the_density(ctx, kind, prec, start):
@@ -118,25 +145,16 @@ def test_captured_solves_follow_the_contrast_of_the_density(ctx, kind, prec, sta
     contrast was there: its replays fall back to multigrid on the device."""
     import kielflow_amd as kf
     print("captured contrast", kind, prec, start, flush=True)
-    n, dt = 24, 1e-3
-    axes = axes_for(kind, n)[0]
-    P = kf.KF_MIXED if prec == "mixed" else kf.KF_FP64
-    B = kf.Batch(ctx, [(axes, kf.api.Parameters(1.0, 0.1, 100.0, 0.0, 0.0))], precision=P, dt=dt, nstreams=1)
-    _, nd, mask = kf.setup_host(axes, seed=3, amp=1e-3, Q=-0.1, a=2.0)
-    B.set_fields(0, ctx.to_device(nd), ctx.to_device(mask))
-    F, phi = B.box(0)
-    x = np.cos(np.arange(n) * 2 * np.pi / n)[:, None, None] + np.zeros((n, n, n))
-    mode = np.fft.rfftn(x)
-    for step in range(6 + 110):
-        if step == 6:
-            B.capture(3)
-            assert B.poisson_failures() == 0
-        F[3].copy_from(ctx.to_device(start * mode if step == 0 else F[3].get() + 0.01 * mode))
-        ctx.sync()
-        B.steps(1)
-        B.sync()
-    e = np.exp(phi.get())
-    print("  exp(phi)", e.min(), e.max(), "failures", B.poisson_failures(), flush=True)
-    assert e.max() / e.min() > 3 and np.isfinite(e).all()
-    assert B.poisson_failures() == 0
-    B.close()
+    lo, hi, failures = _grow_contrast(kf, ctx, kind, (24, 24, 24), prec, start, 6 + 110)
+    assert hi / lo > 3 and failures == 0
+
+
+@pytest.mark.parametrize("kind,dims", [("eqst", (128, 96, 96)), ("sist", (128, 96, 96)), ("eqst", (6, 12, 16)),
+                                       ("hyst", (32, 12, 24))])
+def test_captured_fall_back_of_large_and_shallow_boxes(ctx, kind, dims):
+    """More than 2^20 points, where the fall back is level kernels with a one-workgroup tail, and boxes with few
+    levels: replays converge while the contrast grows through the point where direct corrections stall."""
+    import kielflow_amd as kf
+    print("captured fall back", kind, dims, flush=True)
+    lo, hi, failures = _grow_contrast(kf, ctx, kind, dims, "mixed", 0.3, 6 + 60)
+    assert hi / lo > 2 and failures == 0

@@ -168,6 +168,8 @@ int kf_effect_penalization(kf_grid g, const double *mask, double eta, double fix
 int kf_poisson_create(kf_grid g, int precision, int mode, kf_poisson *out);
 int kf_poisson_destroy(kf_poisson p);
 int kf_poisson_set_tolerance(kf_poisson p, double tol);
+/* Newton corrections of a solve; multigrid that takes over from stalled direct
+ * corrections has this many of its own */
 int kf_poisson_set_max_iterations(kf_poisson p, int iters);
 /* multigrid smoothing of the Newton-MG solver: pre/post red-black sweeps per
  * level and sweeps on the coarsest level (defaults 2, 2, 8 in FP64, 2, 3,

@@ -15,7 +15,7 @@
 // 0.1 for a grain in a plasma; a V-cycle 0.1), for one pass of each axis
 // forth and back instead of a V-cycle's sweeps on every level.  Measured
 // against V-cycles (BiCGStab around them on stretched grids): the first solve
-// of a run 6.2 -> 0.90 ms at 192x128x192 equidistant FP64 and 6.3 -> 0.38 ms
+// of a run 6.2 -> 0.94 ms at 192x128x192 equidistant FP64 and 6.5 -> 0.34 ms
 // at 64^3 hyperbolic; an RK4 step 14.8 -> 12.1 ms (256^3 mixed), 26.9 -> 19.4
 // (256^3 FP64), 18.9 -> 7.9 (128^3 sine FP64).
 #pragma once

@@ -70,8 +70,8 @@ class Poisson {
     // Newton corrections by the direct solver of L_h - c (kf_direct.h) where
     // the grid admits it; multigrid takes them elsewhere, with Boltzmann
     // ions, and from where a direct correction leaves too much (exp(phi)
-    // varies by more than a few times over the box)
-    // (like: an FP64 plan of the grid that is there already, or null)
+    // varies by more than about three times over the box's length).
+    // like: an FP64 plan of the grid that is there already, or null
     void init_direct(const fft::Plan<double> *like = nullptr);
     void set_tolerance(double t) { tol_ = t; }
     void set_max_iterations(int m) { max_it_ = m; }
